@@ -38,7 +38,8 @@ struct sk_potential {
   sk::DevBuf<float2> t;                // nslices x N
   std::vector<int> prop_of_slice;      // index into the compact propagators
   std::vector<double> prop_dz;
-  sk::DevBuf<float2> props;            // nprops x nx x nc, scaled by 1/N
+  sk::DevBuf<float2> props;            // nprops x nx x nc, scaled by 1/N; then, where they differ, the fast passes'
+  size_t props_fast = 0;               // where in props the fast passes' own begin (0: they take the same)
   sk::DevBuf<double> aperture;         // N
   sk::DevBuf<double> V;                // nslices x N (atoms form only)
   bool has_values = false;
@@ -577,15 +578,24 @@ void finish_potential(sk_potential& p, const double* V_dev) {
       p.prop_of_slice[j] = it->second;
     }
   }
-  p.props.alloc(p.prop_dz.size() * (size_t)nx * p.nc);
-  // where the two-stage passes run the slice loop, the propagator divides by what they do to each frequency
+  // where the two-stage passes run the slice loop, its propagators divide by what they do to each frequency; the generic
+  // passes (fast_path = 0) have other constants and keep the propagators as they are: at 243 x 243 the gains come to
+  // 2.9e-7 of the intensity a slice, which either path would lose or gain with the other's
   const LinePlan &px = line_plan(nx, s), &py = line_plan(ny, s);
   const double* gx = fast_col_supported(nx, p.nc, kColMid) || reg_length_supported(px.dev) ? nullptr : px.trip_cols.p;
   const double* gy = fast_row_supported(nx, ny, kRowMid) || reg_length_supported(py.dev) ? nullptr : py.trip_rows.p;
-  for (size_t k = 0; k < p.prop_dz.size(); ++k)
-    launch_propagator(nx, ny, p.grid.extent_x, p.grid.extent_y, p.lambda, p.prop_dz[k], p.tilt[0], p.tilt[1],
-                      p.aperture.p, p.keep_d.p, p.nc, 1.0 / double(N), gx,
-                      gy, p.props.p + k * (size_t)nx * p.nc, s);
+  const size_t props = p.prop_dz.size() * (size_t)nx * p.nc;
+  p.props_fast = gx || gy ? props : 0;
+  p.props.alloc(props + p.props_fast);
+  for (size_t k = 0; k < p.prop_dz.size(); ++k) {
+    auto propagator = [&](const double* rows, const double* columns, float2* out) {
+      launch_propagator(nx, ny, p.grid.extent_x, p.grid.extent_y, p.lambda, p.prop_dz[k], p.tilt[0], p.tilt[1],
+                        p.aperture.p, p.keep_d.p, p.nc, 1.0 / double(N), rows, columns,
+                        out + k * (size_t)nx * p.nc, s);
+    };
+    propagator(nullptr, nullptr, p.props.p);
+    if (p.props_fast) propagator(gx, gy, p.props.p + p.props_fast);
+  }
   SK_HIP(hipStreamSynchronize(s));
 }
 
@@ -807,7 +817,7 @@ void slice_loop(const sk_potential& p, int batch, float2* G, bool entry_full, fl
     row_pass(r, batch, fast, s);
     r.ev_start = r.ev_stop = nullptr;
     // column pass of slice j
-    c.P = p.props.p + (size_t)p.prop_of_slice[j] * p.grid.nx * p.nc;
+    c.P = p.props.p + (fast ? p.props_fast : 0) + (size_t)p.prop_of_slice[j] * p.grid.nx * p.nc;
     if (j == p.nslices - 1 && final_col) {
       ColArgs f = *final_col;
       f.P = c.P;
@@ -928,7 +938,7 @@ void run_pipeline(const sk_potential* const* pots, int npots, int npos, int W, i
       for (int j = 0; j < P.nslices; ++j, ++st) {
         LaneDesc& d = descs[(size_t)st * L + l];
         d.t = P.t.p + (size_t)j * N;
-        d.P = P.props.p + (size_t)P.prop_of_slice[j] * nx * P.nc;
+        d.P = P.props.p + P.props_fast + (size_t)P.prop_of_slice[j] * nx * P.nc;
         d.pos = li[m].pos;
         d.count = li[m].count;
         d.acc_off = acc_off;

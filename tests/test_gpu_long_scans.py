@@ -49,3 +49,10 @@ def errors(nx, ny, options):
 def test_bluestein_scans_keep_their_intensity(nx, ny):
     for e in errors(nx, ny, [sk.ExecutionOptions()]):
         assert np.abs(e).max() <= BOUND
+
+
+@pytest.mark.parametrize("nx,ny", [(198, 198), (486, 486)])
+def test_both_paths_of_smooth_scans_keep_their_intensity(nx, ny):
+    """The generic passes have other constants than the two-stage ones: each path's propagators correct its own."""
+    for e in errors(nx, ny, [sk.ExecutionOptions(), sk.ExecutionOptions(fast_path=False)]):
+        assert np.abs(e).max() <= BOUND
