@@ -14,15 +14,16 @@
 //
 //   n = 509: M = 900 where a power of two took 1024; n = 257: 440 (1024); n = 601: 1024 (2048)
 //
-// Bound by vector arithmetic and LDS, four M-point transforms a pass. Milliseconds per launch on an MI355X, row / column
-// pass, against the passes on power-of-two convolutions (register-resident for 257..512, else in LDS):
-//   131^2 (512 positions)  0.063 / 0.051   0.336 / 0.235     613^2 (123)  0.465 / 0.384   2.04 / 1.46
-//   211^2 (512)            0.165 / 0.159   0.564 / 0.371     701^2 (63)   0.420 / 0.468   1.20 / 0.89
-//   347^2 (256)            0.342 / 0.311   0.422 / 0.335     863^2 (123)  1.33 / 1.24     3.24 / 2.28
-//   509^2 (119)            0.286 / 0.235   0.300 / 0.300     1021^2 (88)  1.98 / 1.50     2.80 / 2.03
-// Slower where a launch carries far more waves than the last-level cache holds (the library's plan never does): 509^2 with
-// 4,096 positions takes 11.4 / 9.0 ms, where register-resident passes on 1024 points, which prefetched each position's
-// loads, took 8.8 / 7.3 ms.
+// Bound by vector arithmetic and LDS, four M-point transforms a pass (509: two wavefronts a SIMD, issuing vector
+// instructions about 80 % of the row pass's time). A unit's loads are issued together, before any is used: where each
+// was used under its slot's condition the compiler waited for one before it issued the next, 2.44 / 1.97 us a position at
+// 509^2 against 2.09 / 1.62, and 2.80 / 2.21 against 2.06 / 1.52 where the waves come from HBM (4,096 positions a launch).
+// Milliseconds per launch on an MI355X, row / column pass, against the passes on power-of-two convolutions that were
+// here before (register-resident for 257..512, else in LDS):
+//   131^2 (512 positions)  0.066 / 0.049   0.336 / 0.235     613^2 (123)   0.379 / 0.316   2.04 / 1.46
+//   211^2 (512)            0.164 / 0.138   0.564 / 0.371     863^2 (123)   1.02 / 0.96     3.24 / 2.28
+//   347^2 (256)            0.297 / 0.234   0.422 / 0.335     1021^2 (88)   1.47 / 1.12     2.80 / 2.03
+//   509^2 (119)            0.249 / 0.193   0.300 / 0.300     509^2 (4096)  8.4 / 6.2       8.8 / 7.3
 #pragma once
 
 #include "sk_pair.h"
@@ -115,18 +116,22 @@ __global__ void __launch_bounds__(PairShape<M>::NT, PairShape<M>::ROW_WAVES) row
     float2* g = a.G + b * gw + (long long)x * a.nc;
     float2 u[RA];
     const int high = M - n + a.kept_shift;  // compact column of a high slot: slot - high
+    // every load first (a slot without a value reads the line's first), then the chirp and the zeros
 #pragma unroll
     for (int r = 0; r < RA; ++r) {
       const int group = blue_group<M>(r), s = il + RB * r;
-      u[r] = make_float2(0.f, 0.f);
-      if (group == PAIR_LOW) {
-        const bool in = s <= a.kept_hi;
-        const float2 t = cmulc(g[in ? s : 0], f.chirp[in ? s : 0]);
-        if (in) u[r] = t;
-      } else if (group == PAIR_HIGH) {
-        const bool in = s >= M - n + a.kept_lo;
-        const float2 t = cmulc(g[in ? s - high : 0], f.chirp[in ? M - s : 0]);
-        if (in) u[r] = t;
+      if (group == PAIR_LOW) u[r] = g[s <= a.kept_hi ? s : 0];
+      if (group == PAIR_HIGH) u[r] = g[s >= M - n + a.kept_lo ? s - high : 0];
+    }
+#pragma unroll
+    for (int r = 0; r < RA; ++r) {
+      const int group = blue_group<M>(r), s = il + RB * r;
+      if (group == PAIR_BAND) {
+        u[r] = make_float2(0.f, 0.f);
+      } else {
+        const bool in = group == PAIR_LOW ? s <= a.kept_hi : s >= M - n + a.kept_lo;
+        const float2 z = cmulc(u[r], f.chirp[in ? (group == PAIR_LOW ? s : M - s) : 0]);
+        u[r] = in ? z : make_float2(0.f, 0.f);
       }
     }
     blue_convolve<M, 1>(u, bi, bq, on_i, on_q, tab + ql, f.inverse + ql);
@@ -202,14 +207,18 @@ __global__ void __launch_bounds__(PairShape<M>::CT, PairShape<M>::COL_WAVES) col
     const unsigned start = live ? unsigned(ni * gw + cb) * 8u : 0u, row = unsigned(a.nc) * 8u;
     auto at = [&](int x) -> float2& { return *reinterpret_cast<float2*>(base + (start + unsigned(x) * row)); };
     float2 u[RA];
+    // as in the row pass: every load first, then the chirp and the zeros
+#pragma unroll
+    for (int r = 0; r < RA; ++r)
+      if (RB * r < NMAX) u[r] = at(live && il + RB * r < n ? il + RB * r : 0);
 #pragma unroll
     for (int r = 0; r < RA; ++r) {
       const int s = il + RB * r;
-      u[r] = make_float2(0.f, 0.f);
       if (RB * r < NMAX) {
-        const bool in = live && s < n;
-        const float2 t = cmul(at(in ? s : 0), f.chirp[in ? s : 0]);
-        if (in) u[r] = t;
+        const float2 z = cmul(u[r], f.chirp[s < n ? s : 0]);
+        u[r] = live && s < n ? z : make_float2(0.f, 0.f);
+      } else {
+        u[r] = make_float2(0.f, 0.f);
       }
     }
     blue_convolve<M, TC>(u, bi, bq, on_i, on_q, tab + ql, f.forward + ql);
