@@ -86,7 +86,9 @@ __host__ __device__ constexpr int blue_group(int r) {
   return RB * r <= H ? PAIR_LOW : RB * (r + 1) - 1 >= M - H ? PAIR_HIGH : PAIR_BAND;
 }
 
-// Row pass: compact line -> inverse [-> exit plane] [-> * t -> forward -> compact line].
+// Row pass: compact line -> inverse [-> exit plane] [-> * t -> forward -> compact line], or a full-width wave -> * t ->
+// forward -> compact line. Only the band of that forward transform is used, so the band's convolution does: one wave of
+// 509^2 enters in 11.7 us, against 26.9 through the 1024 points that every frequency takes.
 template <int M>
 __global__ void __launch_bounds__(PairShape<M>::NT, PairShape<M>::ROW_WAVES) row_blue_kernel(RowArgs a, BlueLine f,
                                                                                            int batch, int rounds) {
@@ -116,44 +118,61 @@ __global__ void __launch_bounds__(PairShape<M>::NT, PairShape<M>::ROW_WAVES) row
     float2* g = a.G + b * gw + (long long)x * a.nc;
     float2 u[RA];
     const int high = M - n + a.kept_shift;  // compact column of a high slot: slot - high
-    // every load first (a slot without a value reads the line's first), then the chirp and the zeros
+    const float2* t = a.t + (long long)x * n;
+    if (a.flags & ROW_INV) {
+      // every load first (a slot without a value reads the line's first), then the chirp and the zeros
 #pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const int group = blue_group<M>(r), s = il + RB * r;
-      if (group == PAIR_LOW) u[r] = g[s <= a.kept_hi ? s : 0];
-      if (group == PAIR_HIGH) u[r] = g[s >= M - n + a.kept_lo ? s - high : 0];
-    }
-#pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const int group = blue_group<M>(r), s = il + RB * r;
-      if (group == PAIR_BAND) {
-        u[r] = make_float2(0.f, 0.f);
-      } else {
-        const bool in = group == PAIR_LOW ? s <= a.kept_hi : s >= M - n + a.kept_lo;
-        const float2 z = cmulc(u[r], f.chirp[in ? (group == PAIR_LOW ? s : M - s) : 0]);
-        u[r] = in ? z : make_float2(0.f, 0.f);
+      for (int r = 0; r < RA; ++r) {
+        const int group = blue_group<M>(r), s = il + RB * r;
+        if (group == PAIR_LOW) u[r] = g[s <= a.kept_hi ? s : 0];
+        if (group == PAIR_HIGH) u[r] = g[s >= M - n + a.kept_lo ? s - high : 0];
       }
-    }
-    blue_convolve<M, 1>(u, bi, bq, on_i, on_q, tab + ql, f.inverse + ql);
-    if ((a.flags & ROW_WRITE_PLANE) && live) {
-      float2* pl = a.plane + b * a.plane_stride + (long long)x * n;
+#pragma unroll
+      for (int r = 0; r < RA; ++r) {
+        const int group = blue_group<M>(r), s = il + RB * r;
+        if (group == PAIR_BAND) {
+          u[r] = make_float2(0.f, 0.f);
+        } else {
+          const bool in = group == PAIR_LOW ? s <= a.kept_hi : s >= M - n + a.kept_lo;
+          const float2 z = cmulc(u[r], f.chirp[in ? (group == PAIR_LOW ? s : M - s) : 0]);
+          u[r] = in ? z : make_float2(0.f, 0.f);
+        }
+      }
+      blue_convolve<M, 1>(u, bi, bq, on_i, on_q, tab + ql, f.inverse + ql);
+      if ((a.flags & ROW_WRITE_PLANE) && live) {
+        float2* pl = a.plane + b * a.plane_stride + (long long)x * n;
+#pragma unroll
+        for (int r = 0; r < RA; ++r) {
+          const int s = il + RB * r;
+          if (RB * r < NMAX && s < n) pl[s] = cscale(cmulc(u[r], f.chirp[s]), a.out_scale);
+        }
+      }
+      if (!(a.flags & ROW_FWD)) continue;
+      // the inverse's closing chirp and the forward's opening one cancel; t is taken as zero past n
 #pragma unroll
       for (int r = 0; r < RA; ++r) {
         const int s = il + RB * r;
-        if (RB * r < NMAX && s < n) pl[s] = cscale(cmulc(u[r], f.chirp[s]), a.out_scale);
+        if (RB * r >= NMAX) {
+          u[r] = make_float2(0.f, 0.f);
+        } else {
+          const float2 p = cmul(u[r], t[s < n ? s : 0]);
+          u[r] = s < n ? p : make_float2(0.f, 0.f);
+        }
       }
-    }
-    if (!(a.flags & ROW_FWD)) continue;
-    // the inverse's closing chirp and the forward's opening one cancel; t is taken as zero past n
-    const float2* t = a.t + (long long)x * n;
+    } else {  // a full-width wave in real space
+      const float2* in = a.in_full + b * a.in_full_stride + (long long)x * n;
 #pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const int s = il + RB * r;
-      if (RB * r >= NMAX) {
-        u[r] = make_float2(0.f, 0.f);
-      } else {
-        const float2 p = cmul(u[r], t[s < n ? s : 0]);
-        u[r] = s < n ? p : make_float2(0.f, 0.f);
+      for (int r = 0; r < RA; ++r)
+        if (RB * r < NMAX) u[r] = in[il + RB * r < n ? il + RB * r : 0];
+#pragma unroll
+      for (int r = 0; r < RA; ++r) {
+        const int s = il + RB * r, sx = s < n ? s : 0;
+        if (RB * r >= NMAX) {
+          u[r] = make_float2(0.f, 0.f);
+        } else {
+          const float2 p = cmul(cmul(u[r], t[sx]), f.chirp[sx]);
+          u[r] = s < n ? p : make_float2(0.f, 0.f);
+        }
       }
     }
     blue_convolve<M, 1>(u, bi, bq, on_i, on_q, tab + ql, f.forward + ql);
