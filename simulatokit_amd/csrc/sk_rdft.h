@@ -53,6 +53,10 @@ constexpr double sin_of(int m, int r) { return cos_of((4 * (m % r) + 3 * r) % (4
 // the errors of the constants' rounding would add up: the way back (BACK) takes other roundings that cancel them as far
 // as float32 goes. For a composite radix, whose roots are factors: the reciprocal conjugates of the first table's
 // entries. For an odd prime, whose sines and cosines are summed: 2 x - (the first table's rounding of x).
+// The cosines of an odd prime sum to -1/2 over half a turn, and so do their roundings here: what they miss (9e-8 for 13,
+// each rounded by itself) would turn a constant line, the bulk of a wave that entered as a plane one, into other
+// frequencies, the same way in every slice. The smallest cosine, which has the finest steps, takes the difference. Exit
+// waves at lengths with a factor 7, 11 or 13 come to 0.72 of their error with it (geometric mean of 47 planes).
 template <int R, bool BACK = false>
 struct RootTable {
   float c[R], s[R];
@@ -64,6 +68,15 @@ struct RootTable {
       const double n = double(c0) * c0 + double(s0) * s0;
       c[m] = !BACK ? c0 : float(prime ? 2 * cx - c0 : c0 / n);
       s[m] = !BACK ? s0 : float(prime ? 2 * sx - s0 : s0 / n);
+    }
+    if (prime && R > 5) {  // 3: -1/2 itself; 5: written as -1/4 +- sqrt(5) / 4
+      int least = 1;
+      double sum = c[1];
+      for (int m = 2; m <= R / 2; ++m) {
+        sum += c[m];
+        if ((c[m] < 0 ? -c[m] : c[m]) < (c[least] < 0 ? -c[least] : c[least])) least = m;
+      }
+      c[least] = c[R - least] = float(c[least] - (sum + 0.5));
     }
   }
 };
