@@ -717,8 +717,8 @@ int sk_separable_map(const float* in, int batch, int n, const float* A, int m, f
     hipStream_t s = pick(stream);
     // tmp[b][v][i] = sum_j in[b][i][j] A[v][j], then out[b][u][v] = sum_i tmp[b][v][i] A[u][i]
     const unsigned tn = (n + kSepTile - 1) / kSepTile, tm = (m + kSepTile - 1) / kSepTile;
-    for (int b0 = 0; b0 < batch; b0 += 65535) {  // the grid's limit of images
-      const unsigned nb = batch - b0 < 65535 ? batch - b0 : 65535;
+    for (long long b0 = 0; b0 < batch; b0 += 65535) {  // the grid's limit of images
+      const unsigned nb = unsigned(batch - b0 < 65535 ? batch - b0 : 65535);
       hipLaunchKernelGGL(sep_half_kernel, dim3(tn, tm, nb), dim3(256), 0, s, in + (size_t)b0 * n * n, A, n, n, m,
                          tmp + (size_t)b0 * n * m);
       hipLaunchKernelGGL(sep_half_kernel, dim3(tm, tm, nb), dim3(256), 0, s, tmp + (size_t)b0 * n * m, A, m, n, m,
