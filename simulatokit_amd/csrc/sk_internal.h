@@ -317,8 +317,8 @@ constexpr size_t kCachedWaveBytes = size_t(240) << 20;
 // columns per block the fast column pass uses for a request of 0, 8 or 16 and a batch of `wave_bytes` compact waves
 int fast_col_tile(int nx, int requested, double wave_bytes);
 int fast_col_blocks_per_wave(int nx, int nc, int pipeline);  // blocks of the detecting column pass per wave
-// register-resident passes for lines of 384 and 1024 points and Bluestein's lengths 257..512 on 1024 points
-// (sk_reg.hip): the row modes of the fast passes, and the middle slices' column pass
+// register-resident passes for lines of 384 and 1024 points (sk_reg.hip): the row modes of the fast passes, and the
+// first, middle and last slices' column passes
 bool reg_length_supported(const LineFFT& f);
 bool reg_row_supported(const RowArgs& a);
 bool reg_col_supported(const ColArgs& a);

@@ -18,7 +18,7 @@
 //
 // Bounds at 600^2 (128 positions, waves in the last-level cache): the row pass issues about 76 vector instructions per
 // point, 0.10 ms at 2.2 GHz of the 0.129 ms it takes; the column pass moves its 0.49 GB at 4.0 TB/s. The Stockham
-// passes it replaces took 0.70 and 0.47 ms: 92 k -> 389 k position-slices/s.
+// passes it replaces took 0.70 and 0.47 ms. A scan of 256 positions and 20 slices: 92 k -> 471 k position-slices/s.
 //
 // A unit of a row pass is one row x of one position; consecutive lines of a block take consecutive units, positions
 // fastest, so they share the row t(x, .) and a small batch still fills the block. A column pass takes TC compact
@@ -50,8 +50,11 @@ struct PairShape {
   static constexpr int RA = pair_ra(M), RB = M / RA;
   static constexpr int S1 = RB | 1;  // LDS row stride: odd, so that lanes q reading column i fall on distinct banks
   static constexpr int LS = RA * S1;
-  // wavefronts per SIMD the registers are held to. 600 (25 x 24): row pass 0.129 ms per 128 positions at three (168
-  // VGPRs) against 0.159 at two; column pass 0.123 against 0.387 ms at three, where P's values spill.
+  // wavefronts per SIMD the registers are held to, by the larger radix. 400 points' columns and the row passes of 546,
+  // 572, 576, 624, 648, 650, 675, 676, 702 and 729 spill 12 to 84 bytes a lane at three; at two the columns of 819 and
+  // more spill up to 128. Where the LDS holds fewer wavefronts than that, the compiler takes the registers that they
+  // leave (600: row pass 177 VGPRs, two). 600's column pass: 0.123 ms per 128 positions at two, 0.387 at three, where P's
+  // values spill.
   static constexpr int ROW_WAVES = RA <= 28 ? 3 : 2, COL_WAVES = RA <= 20 ? 3 : 2;
   // The wavefronts of blocks of `threads` threads that a CU holds (160 KB of LDS with the roots' tables, `waves` per
   // SIMD).

@@ -142,7 +142,6 @@ constexpr int split_of(int r) {
     case 8: return 2;
     case 16: return 4;
     case 32: return 4;
-    case 64: return 8;
     default: break;
   }
   for (int p = 3; p < r; ++p)

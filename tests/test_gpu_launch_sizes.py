@@ -62,3 +62,17 @@ def test_large_launches_cost_no_more_a_position(n, cached, large):
 
     assert per_position(large) <= 1.2 * per_position(cached)
     prepared.release()
+
+
+@pytest.mark.parametrize("nx,ny", [(131, 131), (600, 97), (96, 225)])
+def test_graph_replays_give_the_same_bits(nx, ny):
+    # 11 positions in batches of 4: the second full batch replays the graph that was captured beside the first
+    probe, prepared = scan_of(nx, ny)
+    positions = np.random.default_rng(ny).uniform(0, SRTIO3_A, (11, 2))
+    dets = [sk.AnnularDetector(20, 60), sk.CenterOfMassDetector("cutoff", "mrad"), sk.PixelatedDetector("cutoff")]
+    eager = sk.STEM.scan(probe, [prepared], positions, dets, sk.ExecutionOptions(batch=4))
+    for _ in range(2):
+        replayed = sk.STEM.scan(probe, [prepared], positions, dets, sk.ExecutionOptions(batch=4, use_graph=True))
+        for a, b in zip(eager, replayed):
+            assert np.array_equal(np.asarray(a.values), np.asarray(b.values))
+    prepared.release()
