@@ -18,7 +18,7 @@
 //
 // Bounds at 600^2 (128 positions, waves in the last-level cache): the row pass issues about 76 vector instructions per
 // point, 0.10 ms at 2.2 GHz of the 0.129 ms it takes; the column pass moves its 0.49 GB at 4.0 TB/s. The Stockham
-// passes it replaces took 0.70 and 0.47 ms. A scan of 256 positions and 20 slices: 92 k -> 471 k position-slices/s.
+// passes it replaces took 0.70 and 0.47 ms. A scan of 256 positions and 20 slices: 92 k -> 469 k position-slices/s.
 //
 // A unit of a row pass is one row x of one position; consecutive lines of a block take consecutive units, positions
 // fastest, so they share the row t(x, .) and a small batch still fills the block. A column pass takes TC compact
