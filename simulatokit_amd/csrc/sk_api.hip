@@ -38,8 +38,8 @@ struct sk_potential {
   sk::DevBuf<float2> t;                // nslices x N
   std::vector<int> prop_of_slice;      // index into the compact propagators
   std::vector<double> prop_dz;
-  sk::DevBuf<float2> props;            // nprops x nx x nc, scaled by 1/N; then, where they differ, the fast passes'
-  size_t props_fast = 0;               // where in props the fast passes' own begin (0: they take the same)
+  sk::DevBuf<float2> props;            // nprops x nx x nc, scaled by 1/N
+  sk::DevBuf<float2> props_fast;       // the fast passes' own, where theirs differ
   sk::DevBuf<double> aperture;         // N
   sk::DevBuf<double> V;                // nslices x N (atoms form only)
   bool has_values = false;
@@ -552,18 +552,6 @@ void finish_potential(sk_potential& p, const double* V_dev) {
   p.keepinv_d.upload(p.keepinv, s);
   p.aperture.alloc(N);
   launch_antialias(nx, ny, p.grid.extent_x, p.grid.extent_y, p.aperture.p, s);
-  // t = IFFT2(FFT2(e^{i sigma V}) * A) (Multislice.swift:83-103), in chunks of slices
-  p.t.alloc((size_t)p.nslices * N);
-  DevBuf<float2> A;
-  A.alloc(N);
-  const SplitScale inv_n = split_inverse(double(N));
-  launch_aperture_as_complex(nx, ny, p.aperture.p, inv_n.first, A.p, s);
-  for (int j = 0; j < p.nslices; ++j) launch_phase_to_complex(V_dev + j * N, p.sigma, p.t.p + j * N, N, s);
-  const int chunk = std::max<int>(1, (int)std::min<size_t>(p.nslices, (size_t(512) << 20) / (N * sizeof(float2))));
-  for (int j0 = 0; j0 < p.nslices; j0 += chunk) {
-    const int cnt = std::min(chunk, p.nslices - j0);
-    fft2_batch(p.t.p + (size_t)j0 * N, nx, ny, cnt, -1, A.p, inv_n.second, s);
-  }
   // propagators per distinct thickness (Multislice.swift:136, 145-148), compact, scaled by 1/N
   std::map<double, int> index;
   p.prop_of_slice.resize(p.nslices);
@@ -584,9 +572,23 @@ void finish_potential(sk_potential& p, const double* V_dev) {
   const LinePlan &px = line_plan(nx, s), &py = line_plan(ny, s);
   const double* gx = fast_col_supported(nx, p.nc, kColMid) || reg_length_supported(px.dev) ? nullptr : px.trip_cols.p;
   const double* gy = fast_row_supported(nx, ny, kRowMid) || reg_length_supported(py.dev) ? nullptr : py.trip_rows.p;
+  // t = IFFT2(FFT2(e^{i sigma V}) * A) (Multislice.swift:83-103), in chunks of slices
+  p.t.alloc((size_t)p.nslices * N);
   const size_t props = p.prop_dz.size() * (size_t)nx * p.nc;
-  p.props_fast = gx || gy ? props : 0;
-  p.props.alloc(props + p.props_fast);
+  DevBuf<float2> A;
+  A.alloc(gx || gy ? std::max(N, props) : N);
+  const SplitScale inv_n = split_inverse(double(N));
+  launch_aperture_as_complex(nx, ny, p.aperture.p, inv_n.first, A.p, s);
+  for (int j = 0; j < p.nslices; ++j) launch_phase_to_complex(V_dev + j * N, p.sigma, p.t.p + j * N, N, s);
+  const int chunk = std::max<int>(1, (int)std::min<size_t>(p.nslices, (size_t(512) << 20) / (N * sizeof(float2))));
+  for (int j0 = 0; j0 < p.nslices; j0 += chunk) {
+    const int cnt = std::min(chunk, p.nslices - j0);
+    fft2_batch(p.t.p + (size_t)j0 * N, nx, ny, cnt, -1, A.p, inv_n.second, s);
+  }
+  p.props.alloc(props);
+  // the fast passes' take A's memory, which t is done with (on the same stream): an allocation costs up to 0.3 ms of the
+  // 2 ms of a preparation
+  if (gx || gy) p.props_fast = std::move(A);
   for (size_t k = 0; k < p.prop_dz.size(); ++k) {
     auto propagator = [&](const double* rows, const double* columns, float2* out) {
       launch_propagator(nx, ny, p.grid.extent_x, p.grid.extent_y, p.lambda, p.prop_dz[k], p.tilt[0], p.tilt[1],
@@ -594,7 +596,7 @@ void finish_potential(sk_potential& p, const double* V_dev) {
                         out + k * (size_t)nx * p.nc, s);
     };
     propagator(nullptr, nullptr, p.props.p);
-    if (p.props_fast) propagator(gx, gy, p.props.p + p.props_fast);
+    if (p.props_fast.p) propagator(gx, gy, p.props_fast.p);
   }
   SK_HIP(hipStreamSynchronize(s));
 }
@@ -729,6 +731,12 @@ int detect_blocks_per_wave(const sk_potential& p0, bool fast, int pipe, hipStrea
   return (p0.nc + gcols - 1) / gcols;
 }
 
+// The compact propagator of slice j for the passes that run it.
+const float2* slice_propagator(const sk_potential& p, int j, bool fast) {
+  const float2* props = fast && p.props_fast.p ? p.props_fast.p : p.props.p;
+  return props + (size_t)p.prop_of_slice[j] * p.grid.nx * p.nc;
+}
+
 // Runs `batch` waves whose first row pass input is ready (full real-space waves in `full`, or compact G after a
 // generated INIT); writes requested planes. planes_mask[j] = output index for plane j (or -1).
 struct Timer {
@@ -817,7 +825,7 @@ void slice_loop(const sk_potential& p, int batch, float2* G, bool entry_full, fl
     row_pass(r, batch, fast, s);
     r.ev_start = r.ev_stop = nullptr;
     // column pass of slice j
-    c.P = p.props.p + (fast ? p.props_fast : 0) + (size_t)p.prop_of_slice[j] * p.grid.nx * p.nc;
+    c.P = slice_propagator(p, j, fast);
     if (j == p.nslices - 1 && final_col) {
       ColArgs f = *final_col;
       f.P = c.P;
@@ -938,7 +946,7 @@ void run_pipeline(const sk_potential* const* pots, int npots, int npos, int W, i
       for (int j = 0; j < P.nslices; ++j, ++st) {
         LaneDesc& d = descs[(size_t)st * L + l];
         d.t = P.t.p + (size_t)j * N;
-        d.P = P.props.p + P.props_fast + (size_t)P.prop_of_slice[j] * nx * P.nc;
+        d.P = slice_propagator(P, j, true);
         d.pos = li[m].pos;
         d.count = li[m].count;
         d.acc_off = acc_off;
