@@ -50,7 +50,7 @@ struct PairShape {
   static constexpr int RA = pair_ra(M), RB = M / RA;
   static constexpr int S1 = RB | 1;  // LDS row stride: odd, so that lanes q reading column i fall on distinct banks
   static constexpr int LS = RA * S1;
-  // wavefronts per SIMD the registers are held to, by the larger radix. 400 points' columns and the row passes of 546,
+  // wavefronts per SIMD the registers are held to, by the larger radix. The columns of 360 and 400 points and the row passes of 546,
   // 572, 576, 624, 648, 650, 675, 676, 702 and 729 spill 12 to 84 bytes a lane at three; at two the columns of 819 and
   // more spill up to 128. Where the LDS holds fewer wavefronts than that, the compiler takes the registers that they
   // leave (600: row pass 177 VGPRs, two). 600's column pass: 0.123 ms per 128 positions at two, 0.387 at three, where P's
