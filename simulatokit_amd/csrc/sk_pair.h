@@ -50,11 +50,11 @@ struct PairShape {
   static constexpr int RA = pair_ra(M), RB = M / RA;
   static constexpr int S1 = RB | 1;  // LDS row stride: odd, so that lanes q reading column i fall on distinct banks
   static constexpr int LS = RA * S1;
-  // wavefronts per SIMD the registers are held to, by the larger radix. The columns of 360 and 400 points and the row passes of 546,
-  // 572, 576, 624, 648, 650, 675, 676, 702 and 729 spill 12 to 84 bytes a lane at three; at two the columns of 819 and
-  // more spill up to 128. Where the LDS holds fewer wavefronts than that, the compiler takes the registers that they
-  // leave (600: row pass 177 VGPRs, two). 600's column pass: 0.123 ms per 128 positions at two, 0.387 at three, where P's
-  // values spill.
+  // wavefronts per SIMD the registers are held to, by the larger radix. At three, the columns of 360 and 400 points and
+  // the row passes of 546, 572, 576, 624, 648, 650, 675, 676, 702 and 729 spill 12 to 84 bytes a lane; at two, the columns
+  // of 819 points and more spill up to 128. Where the LDS holds fewer wavefronts than that, the compiler takes the
+  // registers that they leave (600: row pass 177 VGPRs, two). 600's column pass: 0.123 ms per 128 positions at two, 0.387
+  // at three, where P's values spill.
   static constexpr int ROW_WAVES = RA <= 28 ? 3 : 2, COL_WAVES = RA <= 20 ? 3 : 2;
   // The wavefronts of blocks of `threads` threads that a CU holds (160 KB of LDS with the roots' tables, `waves` per
   // SIMD).
